@@ -653,16 +653,28 @@ __device__ __forceinline__ void gcm_records_body(const GcmCtx* __restrict__ ctx,
             for (uint32_t i = tid - SI_T; i < 512u; i += SI_NT - SI_T) fill(i);
     }
 
-    // This workgroup's share of the records' concatenated rows.
-    const uint64_t G = uint64_t(sch.nrec) * sch.rows;
-    const uint64_t g0 = sch.use_starts ? sch.starts[blockIdx.x] : uint64_t(blockIdx.x) * G / sch.nwg;
-    const uint64_t g1 = sch.use_starts ? sch.starts[blockIdx.x + 1] : (uint64_t(blockIdx.x) + 1) * G / sch.nwg;
-    if (g1 == g0) return;  // an empty share (the whole workgroup: no barrier is pending)
-    const uint32_t r0 = uint32_t(g0 / sch.rows);
-    const uint32_t qa0 = uint32_t(g0 - uint64_t(r0) * sch.rows);
-    const uint32_t qb0 = g1 - uint64_t(r0) * sch.rows < sch.rows ? uint32_t(g1 - uint64_t(r0) * sch.rows) : sch.rows;
-    const uint32_t nseg = g1 > (uint64_t(r0) + 1) * sch.rows ? 2u : 1u;
-    const uint32_t qb1 = uint32_t(g1 - (uint64_t(r0) + 1) * sch.rows);  // segment 1: rows [0, qb1) of r0 + 1
+    // This workgroup's share of the records' concatenated rows: rows
+    // [qa0, qb0) of record r0 and, with two segments, [0, qb1) of r0 + 1.  The
+    // laid-out starts are 32-bit, so their record takes a 32-bit division (the
+    // emulated 64-bit one sat on the set-up's critical path); the 64-bit form
+    // is for batches of more than SI_MAX_WG shares only.
+    uint32_t r0, qa0, len;
+    if (sch.use_starts) {
+        const uint32_t g0 = sch.starts[blockIdx.x];
+        len = sch.starts[blockIdx.x + 1] - g0;
+        r0 = g0 / sch.rows;
+        qa0 = g0 - r0 * sch.rows;
+    } else {
+        const uint64_t G = uint64_t(sch.nrec) * sch.rows;
+        const uint64_t g0 = uint64_t(blockIdx.x) * G / sch.nwg;
+        len = uint32_t((uint64_t(blockIdx.x) + 1) * G / sch.nwg - g0);
+        r0 = uint32_t(g0 / sch.rows);
+        qa0 = uint32_t(g0 - uint64_t(r0) * sch.rows);
+    }
+    if (len == 0) return;  // an empty share (the whole workgroup: no barrier is pending)
+    const uint32_t nseg = qa0 + len > sch.rows ? 2u : 1u;
+    const uint32_t qb0 = nseg == 2 ? sch.rows : qa0 + len;
+    const uint32_t qb1 = qa0 + len - sch.rows;
     // Two whole records (the host's pair layout): both segments end at row
     // R, so one placement table serves both.
     const bool pair = nseg == 2 && sch.pairs;
@@ -791,50 +803,54 @@ __device__ __forceinline__ void gcm_records_body(const GcmCtx* __restrict__ ctx,
     // s_barrier does not wait for them.
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (tid < nseg) {
-        const uint32_t s = tid;
+    if (tid < nseg) s_tag[tid] = tag_pre;
+    if (tid < 2 * nseg) {
+        // Lane 2s + h: half h (64 bits) of segment s, so a segment's partial
+        // goes out as one two-lane 64-bit atomic: three atomic operations on
+        // the record's accumulator per share instead of five.  The atomics of
+        // a record's shares queue up on its one line, which bounds a launch
+        // of few records (two 256-KiB records in 44 shares: 2.9 us from the
+        // last barrier to the flags below, of 12.6 us).  MI355X, with the
+        // 32-bit share starts above, four 32-bit XORs -> these: that launch
+        // 13.9 -> 12.6 us, 32 records of 256 KiB 18.4 -> 18.1, 512 of 32 KiB
+        // 28.1 -> 27.7, 96 of 256 KiB 30.3 -> 30.2.
+        const uint32_t s = tid >> 1, h = tid & 1u;
         const uint32_t qa = s ? 0u : qa0, qb = s ? qb1 : qb0;
-        uint32_t r4[4] = {0, 0, 0, 0};
+        const auto half = [&](const uint4* q) { return reinterpret_cast<const uint64_t*>(q)[h]; };
         const uint4* red = (s == 0 && nseg == 2) ? s_c0 : s_red;
+        uint64_t r2 = 0;
 #pragma unroll
-        for (int w = 0; w < SI_NT / 64; ++w) {
-            const uint4 e = red[w];
-            r4[0] ^= e.x; r4[1] ^= e.y; r4[2] ^= e.z; r4[3] ^= e.w;
-        }
-        if (sch.ek_row0 ? qa == 0 : qb == sch.rows) {  // the record's tag mask
-            const uint4 e = s_ek[s];
-            r4[0] ^= e.x; r4[1] ^= e.y; r4[2] ^= e.z; r4[3] ^= e.w;
-        }
-        if (qb == sch.rows) {  // the length block's term
-            r4[0] ^= sch.lh[0]; r4[1] ^= sch.lh[1]; r4[2] ^= sch.lh[2]; r4[3] ^= sch.lh[3];
-        }
+        for (int w = 0; w < SI_NT / 64; ++w) r2 ^= half(red + w);
+        if (sch.ek_row0 ? qa == 0 : qb == sch.rows) r2 ^= half(s_ek + s);  // the record's tag mask
+        if (qb == sch.rows)  // the length block's term
+            r2 ^= h ? uint64_t(sch.lh[3]) << 32 | sch.lh[2] : uint64_t(sch.lh[1]) << 32 | sch.lh[0];
         uint32_t last = 1;
         if (qa != 0 || qb != sch.rows) {
             RecAcc* ra = acc + r0 + s;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                __hip_atomic_fetch_xor(&ra->w[k], r4[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            // Count this segment's rows once its data stores and XORs are
-            // performed.  Write-through stores are complete after s_waitcnt;
-            // byte-granular stores need the agent-scope release (L2 write-back).
-            uint32_t prev;
-            if (kNeedRelease) {
-                prev = __hip_atomic_fetch_add(&ra->count, qb - qa, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-            } else {
-                __builtin_amdgcn_s_waitcnt(0);
-                prev = __hip_atomic_fetch_add(&ra->count, qb - qa, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_xor(&ra->w[h], r2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // Count this segment's rows once its data stores and XORs (both
+            // halves: the wait is the wave's) are performed.  Write-through
+            // stores are complete after s_waitcnt; byte-granular stores need
+            // the agent-scope release (L2 write-back).
+            __builtin_amdgcn_s_waitcnt(0);
+            uint32_t prev = 0;
+            if (h == 0) {
+                if (kNeedRelease)
+                    prev = __hip_atomic_fetch_add(&ra->count, qb - qa, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+                else
+                    prev = __hip_atomic_fetch_add(&ra->count, qb - qa, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             last = prev + (qb - qa) == sch.rows ? 1u : 0u;
-            if (last) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    r4[k] = __hip_atomic_exchange(&ra->w[k], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&ra->count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
         }
-        s_last[s] = last;
-        s_fin[s][0] = r4[0]; s_fin[s][1] = r4[1]; s_fin[s][2] = r4[2]; s_fin[s][3] = r4[3];
-        s_tag[s] = tag_pre;
+        last = uint32_t(__builtin_amdgcn_mov_dpp(int(last), 0xa0, 0xf, 0xf, true));  // lane 2s's: quad_perm [0,0,2,2]
+        if (last && (qa != 0 || qb != sch.rows)) {
+            RecAcc* ra = acc + r0 + s;
+            r2 = __hip_atomic_exchange(&ra->w[h], uint64_t(0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (h == 0) __hip_atomic_store(&ra->count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (h == 0) s_last[s] = last;
+        s_fin[s][2 * h] = uint32_t(r2);
+        s_fin[s][2 * h + 1] = uint32_t(r2 >> 32);
     }
     __syncthreads();
 

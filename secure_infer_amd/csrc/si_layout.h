@@ -31,7 +31,7 @@ struct GcmCtx {
 // One record's cross-workgroup GHASH accumulator; zero between launches
 // (the finalising workgroup resets it).
 struct RecAcc {
-    uint32_t w[4];
+    uint64_t w[2];
     uint32_t count;
     uint32_t reserved[3];
 };

@@ -146,3 +146,22 @@ def test_random_layouts_match_openssl(direction):
     finally:
         si.set_chunk_rows(si.gcm.DEFAULT_CHUNK_ROWS)
         si.set_straddle_rows(si.gcm.DEFAULT_STRADDLE_ROWS)
+
+
+@pytest.mark.parametrize("direction", ["reload", "reload_verify_first", "writeback"])
+@pytest.mark.parametrize("nrec,n,chunk", [(1, 69999, 1), (2, 65536, 1), (768, 4097, 3), (769, 4097, 3)])
+def test_share_starts_and_many_shares_of_a_record(nrec, n, chunk, direction):
+    """The two forms of a share's start (laid out for up to 768 shares,
+    computed in the kernel beyond) on both sides of that limit, and records cut
+    into one-row shares, whose partial sums meet in one accumulator by 64-bit
+    halves.  Against OpenSSL as above."""
+    rng = np.random.default_rng(7500 + nrec)
+    sess = si.GcmSession(KEY, SALT, 0, max_record_bytes=70000)
+    try:
+        si.set_chunk_rows(chunk)
+        if direction == "writeback":
+            _writeback_case(sess, rng, nrec, n, 1)
+        else:
+            _reload_case(sess, rng, nrec, n, 1, strict=direction == "reload_verify_first")
+    finally:
+        si.set_chunk_rows(si.gcm.DEFAULT_CHUNK_ROWS)
