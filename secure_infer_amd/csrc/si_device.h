@@ -309,6 +309,32 @@ __device__ __forceinline__ void gh_fold(const uint4 g[], uint32_t acc[4])
 
 #define SI_STAGE() __builtin_amdgcn_sched_barrier(0)
 
+// Issue priority of a wave with `left` pieces of rows to go (a pair step or a
+// single row; this one included), at the start of a piece and, in the last
+// one, before its GHASH.  The arbiter otherwise favours the oldest wave: it
+// runs one unit's rows to the end while the others wait, then leaves the last
+// unit alone on the SIMDs with too few waves to hide latency.  Each SIMD holds
+// one wave of each unit, so dropping a wave's priority over its last pieces
+// lets the other units catch up.  A segment's start (general rows, counter-mode
+// cache) runs at the highest priority.  MI355X, per layer, against levels by
+// pair steps alone (which left a unit's start, its last pair and its single
+// row at the lowest level; unit 2 of 32 records of 256 KiB ended its rows 3.5
+// us after unit 0): 32 records of 256 KiB 18.2 -> 16.8 us decrypting, 17.6 ->
+// 16.7 encrypting; 512 of 32 KiB 27.9 -> 25.8; int4 4 x 128, 128 records, 22.1
+// -> 21.5; 96 of 256 KiB 30.5 -> 30.4.  A drop inside the last decrypting pair
+// step (its own copy of the step) measured 30.7, 26.3 and 21.9.
+__device__ __forceinline__ void step_priority(uint32_t left)
+{
+    if (left >= 3) __builtin_amdgcn_s_setprio(3);
+    else if (left == 2) __builtin_amdgcn_s_setprio(2);
+    else __builtin_amdgcn_s_setprio(1);
+}
+
+__device__ __forceinline__ void ghash_priority(uint32_t left)
+{
+    if (left == 1) __builtin_amdgcn_s_setprio(0);
+}
+
 // Keystreams of two counter blocks (counter-mode cache of rounds 1-2) and the
 // GHASH fold of a ciphertext row pair, acc = y*H^2T ^ xa*H^T, software
 // pipelined by hand: each stage consumes reads issued two stages earlier and

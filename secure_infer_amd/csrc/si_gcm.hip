@@ -287,7 +287,7 @@ __device__ __forceinline__ void rows_body(const RecView& v, __amdgpu_buffer_rsrc
                                           const AesKeys& keys, const CtrCache& cc, uint32_t n0,
                                           uint32_t n1, uint32_t n2, const uint64_t (&k)[kRows],
                                           const uint4 (&in)[kRows], const uint4 (&ksin)[kRows],
-                                          uint32_t y[4])
+                                          uint32_t left, uint32_t y[4])
 {
     static_assert(kRows == 1 || kRows == 2, "rows per step");
     if constexpr (kRows == 2 && kCached && kMode == MODE_DECRYPT) {
@@ -320,6 +320,7 @@ __device__ __forceinline__ void rows_body(const RecView& v, __amdgpu_buffer_rsrc
         const uint4 xv = kMode == MODE_ENCRYPT ? o[r] : in[r];
         x[r][0] = xv.x; x[r][1] = xv.y; x[r][2] = xv.z; x[r][3] = xv.w;
     }
+    ghash_priority(left);
     if (kRows == 2) {
         uint32_t a[4], b[4];
         gh_mul(gh2, y, a);
@@ -349,19 +350,6 @@ __device__ __forceinline__ void load_rows(const uint4* __restrict__ src, const u
     }
 }
 
-// Issue priority of a wave with `left` pair steps to go (this one included).
-// The arbiter otherwise favours the oldest wave: it runs one unit's rows to
-// the end while the others wait, then leaves the last unit alone on the SIMDs
-// with too few waves to hide latency.  Dropping a step's priority as a wave
-// gets ahead keeps the units of a workgroup within about a step of each other.
-__device__ __forceinline__ void step_priority(uint32_t left)
-{
-    if (left >= 4) __builtin_amdgcn_s_setprio(3);
-    else if (left == 3) __builtin_amdgcn_s_setprio(2);
-    else if (left == 2) __builtin_amdgcn_s_setprio(1);
-    else __builtin_amdgcn_s_setprio(0);
-}
-
 // Full-ciphertext rows i in [i0, i1) of this thread's unit (block k = kb +
 // i*S, S = SI_U*SI_T), two rows per step.  Ping-pong buffers: the loads of
 // the next step are issued before the current step's keystreams, so HBM
@@ -379,6 +367,7 @@ __device__ __forceinline__ void rows_fast(const RecView& v, const uint4* gh, con
     const __amdgpu_buffer_rsrc_t dst = rsrc_of(v.dst);
     const uint32_t nsteps = (i1 - i0) / kP;
     const uint32_t iend = i0 + nsteps * kP;
+    const uint32_t left = nsteps + (iend < i1 ? 1u : 0u);  // pieces: pair steps, then a single row
     if (nsteps) {
         auto rows_of = [&](uint32_t step, uint64_t (&k)[kP]) {
             const uint32_t s = step < nsteps ? step : nsteps - 1;  // clamped prefetch
@@ -393,22 +382,23 @@ __device__ __forceinline__ void rows_fast(const RecView& v, const uint4* gh, con
             rows_of(st + 1, kb2);
             load_rows<kMode, kP>(src, ksrc, kb2, b, qb);
             __builtin_amdgcn_sched_barrier(0);
-            step_priority(nsteps - st);
-            rows_body<kMode, kCached, kP>(v, dst, gh, gh2, aes, lane, keys, cc, n0, n1, n2, ka, a, qa, y);
+            step_priority(left - st);
+            rows_body<kMode, kCached, kP>(v, dst, gh, gh2, aes, lane, keys, cc, n0, n1, n2, ka, a, qa, left - st, y);
             if (st + 1 >= nsteps) break;
             rows_of(st + 2, ka);
             load_rows<kMode, kP>(src, ksrc, ka, a, qa);
             __builtin_amdgcn_sched_barrier(0);
-            step_priority(nsteps - st - 1);
-            rows_body<kMode, kCached, kP>(v, dst, gh, gh2, aes, lane, keys, cc, n0, n1, n2, kb2, b, qb, y);
+            step_priority(left - st - 1);
+            rows_body<kMode, kCached, kP>(v, dst, gh, gh2, aes, lane, keys, cc, n0, n1, n2, kb2, b, qb,
+                                           left - st - 1, y);
         }
-        __builtin_amdgcn_s_setprio(0);
     }
     for (uint32_t i = iend; i < i1; ++i) {
+        step_priority(1);
         uint64_t k1[1] = {kb + uint64_t(i) * kS};
         uint4 a1[1], q1[1];
         load_rows<kMode, 1>(src, ksrc, k1, a1, q1);
-        rows_body<kMode, kCached, 1>(v, dst, gh, gh2, aes, lane, keys, cc, n0, n1, n2, k1, a1, q1, y);
+        rows_body<kMode, kCached, 1>(v, dst, gh, gh2, aes, lane, keys, cc, n0, n1, n2, k1, a1, q1, 1u, y);
     }
 }
 
@@ -475,6 +465,7 @@ __device__ __forceinline__ void unit_rows(const GcmCtx* __restrict__ ctx, const 
     // fast rows) carries the tag-mask job when the batch puts it there.
     uint4* const ek_row = (sch.ek_row0 && qa == 0 && u == 0) ? ek_slot : nullptr;
     y[0] = y[1] = y[2] = y[3] = 0;
+    if (i1 > i0) __builtin_amdgcn_s_setprio(3);  // until the last pieces (step_priority)
     for (uint32_t i = 0; i < i0; ++i) {
         if (i != 0) gh_mul_table(gh, y);
         row_general<kMode, kAligned, kWT>(sch, v, aes, lane, keys, n0, n1, n2,
@@ -500,6 +491,7 @@ __device__ __forceinline__ void unit_rows(const GcmCtx* __restrict__ ctx, const 
             const CtrCache cc{};
             rows_fast<kMode, false>(v, gh, gh2, aes, lane, keys, cc, n0, n1, n2, kb, i0, i1, y);
         }
+        __builtin_amdgcn_s_setprio(0);
     }
     for (uint32_t i = i1; i < nu; ++i) {
         if (i != 0) gh_mul_table(gh, y);
@@ -810,7 +802,7 @@ __device__ __forceinline__ void gcm_records_body(const GcmCtx* __restrict__ ctx,
         // the record's accumulator per share instead of five.  The atomics of
         // a record's shares queue up on its one line, which bounds a launch
         // of few records (two 256-KiB records in 44 shares: 2.9 us from the
-        // last barrier to the flags below, of 12.6 us).  MI355X, with the
+        // last barrier to the flags below, of 13.9 us).  MI355X, with the
         // 32-bit share starts above, four 32-bit XORs -> these: that launch
         // 13.9 -> 12.6 us, 32 records of 256 KiB 18.4 -> 18.1, 512 of 32 KiB
         // 28.1 -> 27.7, 96 of 256 KiB 30.3 -> 30.2.
