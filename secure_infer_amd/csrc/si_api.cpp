@@ -561,6 +561,25 @@ DevCtx* ctx_for(const uint8_t kb[16], const uint8_t hb[16], uint32_t npow)
     return g_ctx_cache.back().get();
 }
 
+// 16 bytes at p and, unless null, at q (device memory) into a and b, after the
+// work on the stream.
+bool read_back(hipStream_t stream, const void* p, uint8_t a[16], const void* q, uint8_t b[16])
+{
+    uint8_t w[32];
+    const hipError_t e = si::fetch_key(stream, p, q, w);
+    if (e == hipErrorNotSupported) {
+        if (hipMemcpyAsync(a, p, 16, hipMemcpyDeviceToHost, stream) != hipSuccess) return false;
+        if (q && hipMemcpyAsync(b, q, 16, hipMemcpyDeviceToHost, stream) != hipSuccess) return false;
+        return hipStreamSynchronize(stream) == hipSuccess;
+    }
+    if (e == hipSuccess) {
+        memcpy(a, w, 16);
+        if (q) memcpy(b, w + 16, 16);
+    }
+    OPENSSL_cleanse(w, sizeof(w));
+    return e == hipSuccess;
+}
+
 // The context of a device-resident key (and H, or zeros): both read back on
 // the stream first.
 DevCtx* ctx_for_device_key(hipStream_t stream, const void* key, const void* h, uint32_t npow)
@@ -570,9 +589,7 @@ DevCtx* ctx_for_device_key(hipStream_t stream, const void* key, const void* h, u
         uint8_t* p;
         ~Cleanse() { OPENSSL_cleanse(p, 16); }
     } cleanse{kb};
-    if (hipMemcpyAsync(kb, key, 16, hipMemcpyDeviceToHost, stream) != hipSuccess) return nullptr;
-    if (h && hipMemcpyAsync(hb, h, 16, hipMemcpyDeviceToHost, stream) != hipSuccess) return nullptr;
-    if (hipStreamSynchronize(stream) != hipSuccess) return nullptr;
+    if (!read_back(stream, key, kb, h, hb)) return nullptr;
     return ctx_for(kb, hb, npow);
 }
 
@@ -581,8 +598,7 @@ DevCtx* ctx_for_hash_subkey(hipStream_t stream, const void* h, uint32_t npow)
 {
     uint8_t hb[16];
     static const uint8_t kZeroKey[16] = {0};
-    if (hipMemcpyAsync(hb, h, 16, hipMemcpyDeviceToHost, stream) != hipSuccess) return nullptr;
-    if (hipStreamSynchronize(stream) != hipSuccess) return nullptr;
+    if (!read_back(stream, h, hb, nullptr, nullptr)) return nullptr;
     return ctx_for(kZeroKey, hb, npow);
 }
 

@@ -166,6 +166,11 @@ hipError_t launch_release(hipStream_t stream, const GcmCtx* ctx, const RecBatch&
                           const LaunchEvents& ev = LaunchEvents());
 hipError_t launch_ctr(hipStream_t stream, const GcmCtx* ctx, const uint8_t* in, uint8_t* out,
                       uint64_t bytes, const uint32_t iv[4]);
+// key[0..16) and, unless null, h[0..16) read by the device after the work on
+// `stream`, into out[0..16) and out[16..32); returns once they are there.
+// hipErrorNotSupported, with nothing queued, for bytes that are not the current
+// device's own memory and for a stream under capture.
+hipError_t fetch_key(hipStream_t stream, const void* key, const void* h, uint8_t out[32]);
 hipError_t launch_auth_gate(hipStream_t stream, uint8_t* data, const uint32_t* status,
                             uint64_t bytes);
 

@@ -15,6 +15,7 @@ typedef enum hipError_t {
     hipErrorInvalidValue = 1,
     hipErrorOutOfMemory = 2,
     hipErrorNotReady = 600,
+    hipErrorNotSupported = 801,
     hipErrorUnknown = 999,
 } hipError_t;
 

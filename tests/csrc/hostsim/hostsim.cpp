@@ -495,6 +495,9 @@ void layer_kernel(int mode, const GcmCtx* ctx, const RecBatch& b, const Sched& s
 
 }  // namespace
 
+// The stand-in has no pinned-memory kernel: the caller copies instead.
+hipError_t fetch_key(hipStream_t, const void*, const void*, uint8_t*) { return hipErrorNotSupported; }
+
 hipError_t launch_gcm(int mode, hipStream_t stream, const GcmCtx* ctx, const RecBatch& b, const Sched& s, RecAcc*,
                       bool, const LaunchEvents&)
 {
