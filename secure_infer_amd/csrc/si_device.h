@@ -447,8 +447,9 @@ __device__ __forceinline__ void be_mulx(uint32_t a[4])
 // z = x * y for per-lane x, y (memory byte order in and out), shared by K
 // threads (K = 2 or 3): Shoup's 4-bit method with a per-lane table of the
 // multiples v*y in LDS.  Each thread writes its share of the table (entries
-// v = c, c+K, ... for c = 0..K-1; v = 0 is not stored: entry v >= 1 sits at
-// tbl[(v - 1) * stride + slot] and a shared zero word stands for v = 0), and
+// v = c, c+K, ... for c = 0..K-1; entry v >= 1 sits at
+// tbl[(v - 1) * stride + slot], and the caller keeps `stride` zero words before
+// tbl as the entries v = 0), and
 // after a barrier each evaluates the nibbles j = c (mod K) of x with its own
 // Horner chain (step x^(4K)), then shifts by x^(4c).  XORing the K results
 // gives x * y; each chain is 1/K as long as one whole product's.
@@ -494,12 +495,11 @@ __device__ __forceinline__ void be_mulx_s(uint32_t a[4])
 // Part C of x * y (C < K) for NS independent products at once (their
 // chains interleave): z[s] = XOR_{j = C mod K} T_s[nibble j of x[s]] * x^(4j),
 // Horner over those nibbles with step x^(4K).  K = 1 is the whole product,
-// K = 2 or 3 a half or a third of it (gh_table_share's layout: entry v >= 1 at
-// tbl[(v - 1) * stride + slot], `zero` for v = 0).
+// K = 2 or 3 a half or a third of it (gh_table_share's layout, the zero words
+// in place: the lookup's address is one shift and add, with no test for 0).
 template <int K, int C, int NS>
 __device__ __forceinline__ void gh_mul_part(const uint32_t (&x_mem)[NS][4], const uint4* const (&tbl)[NS],
-                                            const uint4* zero, uint32_t slot, uint32_t stride,
-                                            uint32_t (&z_mem)[NS][4])
+                                            uint32_t slot, uint32_t stride, uint32_t (&z_mem)[NS][4])
 {
     static_assert((K == 1 || K == 2 || K == 3) && C < K, "one, two or three parts");
     constexpr int kTop = C + K * ((31 - C) / K);
@@ -510,7 +510,7 @@ __device__ __forceinline__ void gh_mul_part(const uint32_t (&x_mem)[NS][4], cons
         for (int k = 0; k < 4; ++k) xb[s][k] = bswap32(x_mem[s][k]);
     const auto entry = [&](int s, int j) -> const uint4* {
         const uint32_t v = (xb[s][j >> 3] >> (28 - 4 * (j & 7))) & 0xfu;
-        return v ? tbl[s] + ((v - 1u) * stride + slot) : zero;
+        return tbl[s] - stride + (v * stride + slot);
     };
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
