@@ -171,6 +171,10 @@ hipError_t launch_ctr(hipStream_t stream, const GcmCtx* ctx, const uint8_t* in, 
 // hipErrorNotSupported, with nothing queued, for bytes that are not the current
 // device's own memory and for a stream under capture.
 hipError_t fetch_key(hipStream_t stream, const void* key, const void* h, uint8_t out[32]);
+// One wave: key[0..16) and, unless null, h[0..16) to out[0..16) and out[16..32),
+// then seq to *flag (out and flag: device addresses of pinned host memory).
+hipError_t launch_key_fetch(hipStream_t stream, const uint8_t* key, const uint8_t* h, uint8_t* out, uint32_t* flag,
+                            uint32_t seq);
 hipError_t launch_auth_gate(hipStream_t stream, uint8_t* data, const uint32_t* status,
                             uint64_t bytes);
 

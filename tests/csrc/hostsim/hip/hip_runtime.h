@@ -40,6 +40,19 @@ typedef enum hipDeviceAttribute_t {
 #define hipEventDefault 0u
 #define hipEventDisableTiming 2u
 #define hipHostMallocDefault 0u
+#define hipHostMallocPortable 1u
+#define hipHostMallocMapped 2u
+
+typedef enum hipMemoryType { hipMemoryTypeHost = 1, hipMemoryTypeDevice = 2 } hipMemoryType;
+
+typedef struct hipPointerAttribute_t {
+    hipMemoryType type;
+    int device;
+} hipPointerAttribute_t;
+
+typedef enum hipStreamCaptureStatus { hipStreamCaptureStatusNone = 0, hipStreamCaptureStatusActive = 1 } hipStreamCaptureStatus;
+
+typedef void* hipDeviceptr_t;
 
 struct uint4 {
     unsigned int x, y, z, w;
@@ -72,6 +85,8 @@ hipError_t hipFreeAsync(void* p, hipStream_t s);
 hipError_t hipHostMalloc(void** p, size_t n, unsigned int flags);
 hipError_t hipHostFree(void* p);
 hipError_t hipHostGetDevicePointer(void** dev, void* host, unsigned int flags);
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p);
+hipError_t hipMemGetAddressRange(hipDeviceptr_t* base, size_t* size, hipDeviceptr_t p);
 hipError_t hipMemcpy(void* dst, const void* src, size_t n, hipMemcpyKind k);
 hipError_t hipMemset(void* p, int v, size_t n);
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind k, hipStream_t s);
@@ -81,6 +96,8 @@ hipError_t hipMemcpy2DAsync(void* dst, size_t dpitch, const void* src, size_t sp
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned int flags);
 hipError_t hipStreamDestroy(hipStream_t s);
 hipError_t hipStreamSynchronize(hipStream_t s);
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* status);
+hipError_t hipLaunchKernel(const void* kernel, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t s);
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned int flags);
 
 hipError_t hipEventCreate(hipEvent_t* e);

@@ -18,6 +18,9 @@
 //   exits:    threads that end inside a layer group and inside a D2H batch;
 //   sessions: a session destroyed while its prefetches are still sealing,
 //             and a destroy refused while another thread holds the session.
+//
+// "key_fetch <what>" runs one scenario of the kernel-level calls' key fetch
+// (si_fetch.cpp) instead.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -35,9 +38,11 @@
 #include <vector>
 
 #include "secure_infer_gpu.h"
+#include "si_kernels.h"
 #include "si_oracle.h"
 
 extern "C" size_t hostsim_reload_log(uint32_t layer, uint64_t* out, size_t cap);
+extern "C" void hostsim_refuse(const char* call);
 
 namespace {
 
@@ -461,8 +466,52 @@ void watchdog(int rounds, int limit)
     }
 }
 
+// ---------------------------------------------------------------- key fetch
+
+// A device-resident key and H: 32 bytes that no other pair shares.
+struct KeyPair {
+    uint8_t bytes[32];
+    uint8_t* dev = nullptr;
+
+    explicit KeyPair(uint32_t seed)
+    {
+        std::mt19937 rng(seed);
+        for (uint8_t& b : bytes) b = uint8_t(rng());
+        CHECK(hipMalloc(&dev, 32) == hipSuccess, "hipMalloc");
+        memcpy(dev, bytes, 32);
+    }
+    ~KeyPair() { (void)hipFree(dev); }
+    hipError_t fetch(hipStream_t s, uint8_t out[32]) const { return si::fetch_key(s, dev, dev + 16, out); }
+    bool fetched(hipStream_t s) const
+    {
+        uint8_t out[32] = {0};
+        return fetch(s, out) == hipSuccess && !memcmp(out, bytes, 32);
+    }
+};
+
+// An earlier call's failure, still the thread's last error, is not the
+// fetch's: the fetch succeeds and leaves the error to its owner.
+void fetch_with_a_pending_error()
+{
+    const KeyPair k(1);
+    void* p = nullptr;
+    hostsim_refuse("hipMalloc");
+    CHECK(hipMalloc(&p, 16) == hipErrorOutOfMemory, "refused");
+    CHECK(k.fetched(nullptr), "fetch beside a pending error");
+    CHECK(hipGetLastError() == hipErrorOutOfMemory, "the error stays pending");
+}
+
 int main(int argc, char** argv)
 {
+    if (argc > 2 && std::string(argv[1]) == "key_fetch") {
+        const std::string what = argv[2];
+        if (what == "pending_error") fetch_with_a_pending_error();
+        else return 2;
+        hipDeviceSynchronize();
+        if (g_failures.load()) return 1;
+        printf("KEY_FETCH_OK\n");
+        return 0;
+    }
     if (argc > 1 && std::string(argv[1]) == "d2h_failure") {
         // One store batch with one record corrupted on its way to the host:
         // the batch fails (batch_end -1, the block zeroed), or, with

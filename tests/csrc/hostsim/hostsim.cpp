@@ -31,10 +31,12 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <string>
 #include <thread>
 #include <vector>
 
 #include "si_kernels.h"
+#include "si_launch.h"
 #include "si_layout.h"
 #include "si_oracle.h"
 
@@ -150,6 +152,65 @@ std::shared_ptr<ihipEvent_t> E(hipEvent_t e)
 
 }  // namespace
 
+namespace {
+
+// Live allocations by address.
+struct Mem {
+    size_t bytes;
+    hipMemoryType type;
+};
+std::mutex g_mem_m;
+std::map<uintptr_t, Mem>& g_mem = *new std::map<uintptr_t, Mem>();
+
+std::map<uintptr_t, Mem>::iterator mem_of(const void* p)
+{
+    const uintptr_t a = reinterpret_cast<uintptr_t>(p);
+    auto it = g_mem.upper_bound(a);
+    if (it == g_mem.begin()) return g_mem.end();
+    --it;
+    return a - it->first < it->second.bytes ? it : g_mem.end();
+}
+
+hipError_t alloc(void** p, size_t n, hipMemoryType type)
+{
+    *p = aligned_alloc(256, (n + 255) / 256 * 256 + 256);
+    if (!*p) return hipErrorOutOfMemory;
+    std::lock_guard<std::mutex> g(g_mem_m);
+    g_mem[reinterpret_cast<uintptr_t>(*p)] = Mem{n, type};
+    return hipSuccess;
+}
+
+void drop(void* p)
+{
+    {
+        std::lock_guard<std::mutex> g(g_mem_m);
+        g_mem.erase(reinterpret_cast<uintptr_t>(p));
+    }
+    free(p);
+}
+
+thread_local hipError_t t_last = hipSuccess;
+
+hipError_t failed(hipError_t e)
+{
+    t_last = e;
+    return e;
+}
+
+// The calling thread's next call of this name fails (hostsim_refuse).
+thread_local std::string t_refused;
+
+bool refused(const char* call)
+{
+    if (t_refused != call) return false;
+    t_refused.clear();
+    return true;
+}
+
+}  // namespace
+
+extern "C" void hostsim_refuse(const char* call) { t_refused = call; }
+
 hipError_t hipGetDevice(int* dev)
 {
     *dev = 0;
@@ -180,35 +241,71 @@ hipError_t hipDeviceSynchronize(void)
     return hipSuccess;
 }
 
-hipError_t hipGetLastError(void) { return hipSuccess; }
+// As HIP keeps it: the thread's last failure, until it is read.
+hipError_t hipGetLastError(void)
+{
+    const hipError_t e = t_last;
+    t_last = hipSuccess;
+    return e;
+}
 
 hipError_t hipMalloc(void** p, size_t n)
 {
-    *p = aligned_alloc(256, (n + 255) / 256 * 256 + 256);
-    return *p ? hipSuccess : hipErrorOutOfMemory;
+    if (refused("hipMalloc")) return failed(hipErrorOutOfMemory);
+    return alloc(p, n, hipMemoryTypeDevice);
 }
 
 hipError_t hipFree(void* p)
 {
-    free(p);
+    drop(p);
     return hipSuccess;
 }
 
-hipError_t hipMallocAsync(void** p, size_t n, hipStream_t) { return hipMalloc(p, n); }
+hipError_t hipMallocAsync(void** p, size_t n, hipStream_t) { return alloc(p, n, hipMemoryTypeDevice); }
 
 hipError_t hipFreeAsync(void* p, hipStream_t s)
 {
-    S(s)->push([p] { free(p); });
+    S(s)->push([p] { drop(p); });
     return hipSuccess;
 }
 
-hipError_t hipHostMalloc(void** p, size_t n, unsigned int) { return hipMalloc(p, n); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned int)
+{
+    if (refused("hipHostMalloc")) return failed(hipErrorOutOfMemory);
+    return alloc(p, n, hipMemoryTypeHost);
+}
 
 hipError_t hipHostFree(void* p) { return hipFree(p); }
 
 hipError_t hipHostGetDevicePointer(void** dev, void* host, unsigned int)
 {
+    if (refused("hipHostGetDevicePointer")) return failed(hipErrorInvalidValue);
     *dev = host;
+    return hipSuccess;
+}
+
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p)
+{
+    std::lock_guard<std::mutex> g(g_mem_m);
+    const auto it = mem_of(p);
+    if (it == g_mem.end()) return failed(hipErrorInvalidValue);
+    *a = hipPointerAttribute_t{it->second.type, 0};
+    return hipSuccess;
+}
+
+hipError_t hipMemGetAddressRange(hipDeviceptr_t* base, size_t* size, hipDeviceptr_t p)
+{
+    std::lock_guard<std::mutex> g(g_mem_m);
+    const auto it = mem_of(p);
+    if (it == g_mem.end()) return failed(hipErrorInvalidValue);
+    *base = reinterpret_cast<void*>(it->first);
+    *size = it->second.bytes;
+    return hipSuccess;
+}
+
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* status)
+{
+    *status = hipStreamCaptureStatusNone;
     return hipSuccess;
 }
 
@@ -263,6 +360,7 @@ hipError_t hipStreamDestroy(hipStream_t s)
 
 hipError_t hipStreamSynchronize(hipStream_t s)
 {
+    if (refused("hipStreamSynchronize")) return failed(hipErrorUnknown);
     S(s)->sync();
     return hipSuccess;
 }
@@ -495,8 +593,22 @@ void layer_kernel(int mode, const GcmCtx* ctx, const RecBatch& b, const Sched& s
 
 }  // namespace
 
-// The stand-in has no pinned-memory kernel: the caller copies instead.
-hipError_t fetch_key(hipStream_t, const void*, const void*, uint8_t*) { return hipErrorNotSupported; }
+// The key fetch's one wave, between its byte stores and its flag a test's hook.
+std::function<void(const uint8_t*)>& g_fetch_hook = *new std::function<void(const uint8_t*)>();
+
+void key_fetch_kernel(const uint8_t* key, const uint8_t* h, uint8_t* out, uint32_t* flag, uint32_t seq)
+{
+    memcpy(out, key, 16);
+    if (h) memcpy(out + 16, h, 16);
+    if (g_fetch_hook) g_fetch_hook(key);
+    __atomic_store_n(flag, seq, __ATOMIC_RELEASE);
+}
+
+hipError_t launch_key_fetch(hipStream_t stream, const uint8_t* key, const uint8_t* h, uint8_t* out, uint32_t* flag,
+                            uint32_t seq)
+{
+    return launch(key_fetch_kernel, dim3(1), dim3(64), stream, key, h, out, flag, seq);
+}
 
 hipError_t launch_gcm(int mode, hipStream_t stream, const GcmCtx* ctx, const RecBatch& b, const Sched& s, RecAcc*,
                       bool, const LaunchEvents&)
@@ -633,6 +745,36 @@ hipError_t launch_blake2b_test(hipStream_t, const uint8_t*, uint32_t, const uint
 }
 
 }  // namespace si
+
+// The one kernel the stand-in launches by its handle.
+hipError_t hipLaunchKernel(const void* kernel, dim3, dim3, void** args, size_t, hipStream_t s)
+{
+    if (kernel != reinterpret_cast<const void*>(&si::key_fetch_kernel)) return failed(hipErrorInvalidValue);
+    const auto key = *static_cast<const uint8_t**>(args[0]);
+    const auto h = *static_cast<const uint8_t**>(args[1]);
+    const auto out = *static_cast<uint8_t**>(args[2]);
+    const auto flag = *static_cast<uint32_t**>(args[3]);
+    const auto seq = *static_cast<uint32_t*>(args[4]);
+    S(s)->push([=] { si::key_fetch_kernel(key, h, out, flag, seq); });
+    return hipSuccess;
+}
+
+// A test's hook in the key fetch (its argument: the fetch's key), set and
+// cleared while no fetch is queued.
+void hostsim_fetch_hook(std::function<void(const uint8_t*)> f) { si::g_fetch_hook = std::move(f); }
+
+// Copies of `n` bytes equal to `b` in pinned host memory.
+size_t hostsim_pinned_copies(const uint8_t* b, size_t n)
+{
+    size_t found = 0;
+    std::lock_guard<std::mutex> g(g_mem_m);
+    for (const auto& m : g_mem) {
+        if (m.second.type != hipMemoryTypeHost) continue;
+        const auto* p = reinterpret_cast<const uint8_t*>(m.first);
+        for (size_t i = 0; i + n <= m.second.bytes; ++i) found += memcmp(p + i, b, n) == 0;
+    }
+    return found;
+}
 
 // Takes the reload log of one layer out of the log (layer numbers come back
 // in later rounds): rows of (kind, block id, ticket); returns the count (at

@@ -1,5 +1,5 @@
 """The host transfer runtime (si_host.cpp, with the session / control code of
-si_api.cpp) under ThreadSanitizer and AddressSanitizer, on the CPU.
+si_api.cpp and the key fetch of si_fetch.cpp) under ThreadSanitizer and AddressSanitizer, on the CPU.
 
 The library's host code is built with g++ against a test-only stand-in for
 the HIP runtime (tests/csrc/hostsim: streams are worker threads, events are
@@ -81,3 +81,13 @@ def test_d2h_authentication_failure_handling(abort):
         assert "D2H_FAILURE_REPORTED" not in r.stdout
     else:
         assert r.returncode == 0 and "D2H_FAILURE_REPORTED" in r.stdout, report[-4000:]
+
+
+@pytest.mark.parametrize("what", ["pending_error"])
+@pytest.mark.parametrize("san", ["thread", "address"])
+def test_key_fetch(san, what):
+    """The host's read of a device-resident key (si_fetch.cpp): an earlier
+    call's pending error does not abandon a queued fetch."""
+    r = subprocess.run([str(build(san)), "key_fetch", what], capture_output=True, text=True, timeout=120,
+                       env={**os.environ, "TSAN_OPTIONS": "halt_on_error=1", "ASAN_OPTIONS": "halt_on_error=1"})
+    assert r.returncode == 0 and "KEY_FETCH_OK" in r.stdout, (r.stdout + r.stderr)[-4000:]
