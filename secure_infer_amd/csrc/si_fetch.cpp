@@ -26,6 +26,52 @@ bool own_device_bytes(const void* p, int dev)
     return off <= size && size - off >= 16;
 }
 
+// Where a fetch lands: pinned memory that the device can write.
+struct Box {
+    uint8_t bytes[32];
+    uint32_t flag;
+};
+
+// The boxes.  One in use at a time (the lock); a fetch whose end was not seen
+// (its stream could not be waited for) may still write its own, so that box is
+// left until its flag shows that the kernel has ended.
+struct Slot {
+    Box* box = nullptr;
+    uint32_t unseen = 0;  // the sequence number of a fetch not seen to end
+};
+constexpr int kSlots = 16;
+std::mutex g_boxes_lock;
+Slot g_boxes[kSlots];
+uint32_t g_seq = 0;  // never 0 in a fetch
+
+bool landed(const Box* b, uint32_t seq) { return __atomic_load_n(&b->flag, __ATOMIC_ACQUIRE) == seq; }
+
+void wipe(Box* b)
+{
+    volatile uint8_t* const w = b->bytes;
+    for (size_t k = 0; k < sizeof(b->bytes); ++k) w[k] = 0;
+}
+
+// A slot that no kernel can write, with its box (nullptr: none free, or no
+// memory).  Unseen fetches that have ended since give theirs back, wiped.
+Slot* take_slot()
+{
+    Slot* free_slot = nullptr;
+    for (Slot& s : g_boxes) {
+        if (s.unseen && landed(s.box, s.unseen)) {
+            wipe(s.box);
+            s.unseen = 0;
+        }
+        if (!s.unseen && (!free_slot || (!free_slot->box && s.box))) free_slot = &s;
+    }
+    if (free_slot && !free_slot->box) {
+        void* b = nullptr;
+        if (hipHostMalloc(&b, sizeof(Box), hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) return nullptr;
+        free_slot->box = new (b) Box();
+    }
+    return free_slot;
+}
+
 }  // namespace
 
 // The kernel-level calls take the key and H as device pointers and need their
@@ -33,17 +79,10 @@ bool own_device_bytes(const void* p, int dev)
 // synchronisation cost such a call about 30 us beyond its record kernel; one
 // wave that stores both into pinned host memory, and a host that watches for
 // its flag, costs a launch and a PCIe write.  MI355X, a 100,003-byte record
-// sealed and then opened: 87.0 -> 40.1 us for the pair.  Only a wait longer than the spin (earlier
-// work on the stream) falls back to synchronising the stream.
+// sealed and then opened: 87.0 -> 40.1 us for the pair.  Only a wait longer than
+// the spin (earlier work on the stream) falls back to synchronising the stream.
 hipError_t fetch_key(hipStream_t stream, const void* key, const void* h, uint8_t out[32])
 {
-    struct Box {
-        uint8_t bytes[32];
-        uint32_t flag;
-    };
-    static std::mutex m;
-    static Box* box = nullptr;
-    static uint32_t seq = 0;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return hipErrorNotSupported;
     if (!own_device_bytes(key, dev) || (h && !own_device_bytes(h, dev))) return hipErrorNotSupported;
@@ -52,33 +91,33 @@ hipError_t fetch_key(hipStream_t stream, const void* key, const void* h, uint8_t
         (void)hipGetLastError();
         return hipErrorNotSupported;
     }
-    std::lock_guard<std::mutex> g(m);
-    if (!box) {
-        void* b = nullptr;
-        if (hipHostMalloc(&b, sizeof(Box), hipHostMallocPortable | hipHostMallocMapped) != hipSuccess)
-            return hipErrorNotSupported;
-        box = new (b) Box();
-    }
+    std::lock_guard<std::mutex> g(g_boxes_lock);
+    Slot* const slot = take_slot();
+    if (!slot) return hipErrorNotSupported;
+    Box* const box = slot->box;
     void* dbox = nullptr;
     hipError_t e = hipHostGetDevicePointer(&dbox, box, 0);
     if (e != hipSuccess) return e;
     Box* const db = static_cast<Box*>(dbox);
-    ++seq;
+    if (++g_seq == 0) g_seq = 1;
+    const uint32_t seq = g_seq;
     e = launch_key_fetch(stream, static_cast<const uint8_t*>(key), static_cast<const uint8_t*>(h), db->bytes, &db->flag,
                          seq);
     if (e != hipSuccess) return e;
     constexpr int kSpins = 20000;
     int i = 0;
-    while (__atomic_load_n(&box->flag, __ATOMIC_ACQUIRE) != seq && ++i < kSpins) __builtin_ia32_pause();
+    while (!landed(box, seq) && ++i < kSpins) __builtin_ia32_pause();
     if (i == kSpins) {
         e = hipStreamSynchronize(stream);
-        if (e == hipSuccess && __atomic_load_n(&box->flag, __ATOMIC_ACQUIRE) != seq) e = hipErrorUnknown;
+        if (!landed(box, seq)) {
+            slot->unseen = seq;
+            return e != hipSuccess ? e : hipErrorUnknown;
+        }
     }
-    volatile uint8_t* const w = box->bytes;
-    for (int k = 0; k < 32; ++k) {
-        if (e == hipSuccess && (k < 16 || h)) out[k] = w[k];
-        w[k] = 0;
-    }
+    const volatile uint8_t* const w = box->bytes;
+    if (e == hipSuccess)
+        for (int k = 0; k < (h ? 32 : 16); ++k) out[k] = w[k];
+    wipe(box);
     return e;
 }
 

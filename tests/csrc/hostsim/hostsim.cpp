@@ -759,6 +759,9 @@ hipError_t hipLaunchKernel(const void* kernel, dim3, dim3, void** args, size_t, 
     return hipSuccess;
 }
 
+// A test's own task on a stream.
+void hostsim_push(hipStream_t s, std::function<void()> f) { S(s)->push(std::move(f)); }
+
 // A test's hook in the key fetch (its argument: the fetch's key), set and
 // cleared while no fetch is queued.
 void hostsim_fetch_hook(std::function<void(const uint8_t*)> f) { si::g_fetch_hook = std::move(f); }
