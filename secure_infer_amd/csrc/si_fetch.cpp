@@ -53,7 +53,7 @@ void wipe(Box* b)
 }
 
 // A slot that no kernel can write, with its box (nullptr: none free, or no
-// memory).  Unseen fetches that have ended since give theirs back, wiped.
+// memory; no error stays pending).  Unseen fetches that have ended since give theirs back, wiped.
 Slot* take_slot()
 {
     Slot* free_slot = nullptr;
@@ -66,7 +66,10 @@ Slot* take_slot()
     }
     if (free_slot && !free_slot->box) {
         void* b = nullptr;
-        if (hipHostMalloc(&b, sizeof(Box), hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) return nullptr;
+        if (hipHostMalloc(&b, sizeof(Box), hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
         free_slot->box = new (b) Box();
     }
     return free_slot;
@@ -84,7 +87,10 @@ Slot* take_slot()
 hipError_t fetch_key(hipStream_t stream, const void* key, const void* h, uint8_t out[32])
 {
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return hipErrorNotSupported;
+    if (hipGetDevice(&dev) != hipSuccess) {
+        (void)hipGetLastError();
+        return hipErrorNotSupported;
+    }
     if (!own_device_bytes(key, dev) || (h && !own_device_bytes(h, dev))) return hipErrorNotSupported;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
@@ -96,13 +102,15 @@ hipError_t fetch_key(hipStream_t stream, const void* key, const void* h, uint8_t
     if (!slot) return hipErrorNotSupported;
     Box* const box = slot->box;
     void* dbox = nullptr;
-    hipError_t e = hipHostGetDevicePointer(&dbox, box, 0);
-    if (e != hipSuccess) return e;
+    if (hipHostGetDevicePointer(&dbox, box, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        return hipErrorNotSupported;
+    }
     Box* const db = static_cast<Box*>(dbox);
     if (++g_seq == 0) g_seq = 1;
     const uint32_t seq = g_seq;
-    e = launch_key_fetch(stream, static_cast<const uint8_t*>(key), static_cast<const uint8_t*>(h), db->bytes, &db->flag,
-                         seq);
+    hipError_t e = launch_key_fetch(stream, static_cast<const uint8_t*>(key), static_cast<const uint8_t*>(h), db->bytes,
+                                    &db->flag, seq);
     if (e != hipSuccess) return e;
     constexpr int kSpins = 20000;
     int i = 0;

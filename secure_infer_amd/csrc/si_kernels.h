@@ -168,8 +168,9 @@ hipError_t launch_ctr(hipStream_t stream, const GcmCtx* ctx, const uint8_t* in, 
                       uint64_t bytes, const uint32_t iv[4]);
 // key[0..16) and, unless null, h[0..16) read by the device after the work on
 // `stream`, into out[0..16) and out[16..32); returns once they are there.
-// hipErrorNotSupported, with nothing queued, for bytes that are not the current
-// device's own memory and for a stream under capture.
+// hipErrorNotSupported, with nothing queued and no error left pending, for bytes
+// that are not the current device's own memory, for a stream under capture and
+// where there is no pinned memory to fetch into.
 hipError_t fetch_key(hipStream_t stream, const void* key, const void* h, uint8_t out[32]);
 // One wave: key[0..16) and, unless null, h[0..16) to out[0..16) and out[16..32),
 // then seq to *flag (out and flag: device addresses of pinned host memory).

@@ -505,6 +505,27 @@ void fetch_with_a_pending_error()
     CHECK(hipGetLastError() == hipErrorOutOfMemory, "the error stays pending");
 }
 
+// No pinned memory, or none the device can address, and bytes that are not the
+// device's: the fetch is declined (the caller copies) and leaves no error.
+void declined_fetches()
+{
+    const KeyPair k(4);
+    uint8_t out[32], host[48] = {0};
+    for (const char* call : {"hipGetDevice", "hipHostMalloc", "hipHostGetDevicePointer"}) {
+        hostsim_refuse(call);
+        CHECK(k.fetch(nullptr, out) == hipErrorNotSupported, "%s refused", call);
+        CHECK(hipGetLastError() == hipSuccess, "%s refused: an error stays pending", call);
+        hostsim_refuse("");
+    }
+    CHECK(k.fetched(nullptr), "a fetch after the refusals");
+    CHECK(si::fetch_key(nullptr, host, nullptr, out) == hipErrorNotSupported, "host memory");
+    CHECK(si::fetch_key(nullptr, k.dev + 17, nullptr, out) == hipErrorNotSupported, "15 bytes left");
+    CHECK(si::fetch_key(nullptr, k.dev, k.dev + 17, out) == hipErrorNotSupported, "H: 15 bytes left");
+    CHECK(hipGetLastError() == hipSuccess, "an error stays pending");
+    CHECK(si::fetch_key(nullptr, k.dev + 16, nullptr, out) == hipSuccess && !memcmp(out, k.bytes + 16, 16),
+          "an allocation's last 16 bytes");
+}
+
 // A fetch on a held stream whose wait fails: its kernel ends during another
 // stream's fetch, after that one stored its key and before its flag.  The second
 // gets its own key, and the first one's does not stay in pinned memory.
@@ -560,6 +581,7 @@ int main(int argc, char** argv)
         const std::string what = argv[2];
         if (what == "pending_error") fetch_with_a_pending_error();
         else if (what == "unseen_end") fetch_not_seen_to_end();
+        else if (what == "declined") declined_fetches();
         else return 2;
         hipDeviceSynchronize();
         if (g_failures.load()) return 1;

@@ -213,6 +213,7 @@ extern "C" void hostsim_refuse(const char* call) { t_refused = call; }
 
 hipError_t hipGetDevice(int* dev)
 {
+    if (refused("hipGetDevice")) return failed(hipErrorUnknown);
     *dev = 0;
     return hipSuccess;
 }
