@@ -25,6 +25,7 @@
 // radix-2^16 limbs in 64-bit integers); BLAKE2b follows RFC 7693 (keyed, 12
 // rounds).  Neither is performance-relevant: they run once per session.
 #include "si_kernels.h"
+#include "si_launch.h"
 #include "si_device.h"
 
 #include <hip/hip_runtime.h>
@@ -502,37 +503,34 @@ hipError_t launch_agree(hipStream_t stream, const uint8_t* host_public, const ui
 {
     constexpr uint32_t kBlocks = 512, kThreads = 256, kRounds = 8;
     static_assert(kBlocks * kThreads == SI_AGREE_POOL_WORDS, "pool size");
-    hipLaunchKernelGGL(zero_bytes_kernel, dim3(1), dim3(64), 0, stream, reinterpret_cast<uint8_t*>(counter), 4u);
-    hipLaunchKernelGGL(entropy_kernel, dim3(kBlocks), dim3(kThreads), 0, stream, pool, counter, kRounds);
-    hipLaunchKernelGGL(agree_kernel, dim3(1), dim3(64), 0, stream, host_public, challenge, seed, pool,
-                       kBlocks * kThreads, key_out, device_public, proof, status);
-    return hipGetLastError();
+    hipError_t e = launch(zero_bytes_kernel, dim3(1), dim3(64), stream, reinterpret_cast<uint8_t*>(counter), 4u);
+    if (e == hipSuccess) e = launch(entropy_kernel, dim3(kBlocks), dim3(kThreads), stream, pool, counter, kRounds);
+    if (e == hipSuccess)
+        e = launch(agree_kernel, dim3(1), dim3(64), stream, host_public, challenge, seed, pool, kBlocks * kThreads,
+                   key_out, device_public, proof, status);
+    return e;
 }
 
 hipError_t launch_ctx_build(hipStream_t stream, const uint8_t* key, const uint32_t* te0, GcmCtx* ctx,
                             uint32_t npow)
 {
-    hipLaunchKernelGGL(ctx_build_kernel, dim3(1), dim3(256), 0, stream, key, te0, ctx, npow);
-    return hipGetLastError();
+    return launch(ctx_build_kernel, dim3(1), dim3(256), stream, key, te0, ctx, npow);
 }
 
 hipError_t launch_zero_bytes(hipStream_t stream, uint8_t* p, uint32_t n)
 {
-    hipLaunchKernelGGL(zero_bytes_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, p, n);
-    return hipGetLastError();
+    return launch(zero_bytes_kernel, dim3((n + 255) / 256), dim3(256), stream, p, n);
 }
 
 hipError_t launch_x25519_test(hipStream_t stream, const uint8_t* scalar, const uint8_t* u, uint8_t* out)
 {
-    hipLaunchKernelGGL(x25519_test_kernel, dim3(1), dim3(64), 0, stream, scalar, u, out);
-    return hipGetLastError();
+    return launch(x25519_test_kernel, dim3(1), dim3(64), stream, scalar, u, out);
 }
 
 hipError_t launch_blake2b_test(hipStream_t stream, const uint8_t* key, uint32_t key_len, const uint8_t* msg,
                                uint64_t msg_len, uint8_t* out, uint32_t out_len)
 {
-    hipLaunchKernelGGL(blake2b_test_kernel, dim3(1), dim3(64), 0, stream, key, key_len, msg, msg_len, out, out_len);
-    return hipGetLastError();
+    return launch(blake2b_test_kernel, dim3(1), dim3(64), stream, key, key_len, msg, msg_len, out, out_len);
 }
 
 }  // namespace si

@@ -20,6 +20,7 @@
 #include "si_codec_math.h"
 #include "si_clock.h"
 #include "si_kernels.h"
+#include "si_launch.h"
 
 namespace si {
 
@@ -502,12 +503,7 @@ hipError_t launch_dequant_scatter(hipStream_t stream, const CodecBatch& b, const
     const dim3 grid(kx * b.n_k + vx * (b.nrec - b.n_k));
     CodecBatch bb = b;
     bb.clock = ev.clock ? ev.clock->take(uint64_t(grid.x) * 4u) : nullptr;
-    if (ev.start || ev.stop)
-        hipExtLaunchKernelGGL(dequant_scatter_kernel, grid, dim3(256), 0, stream, ev.start, ev.stop, 0, bb, kx, vx,
-                              tk, tv);
-    else
-        hipLaunchKernelGGL(dequant_scatter_kernel, grid, dim3(256), 0, stream, bb, kx, vx, tk, tv);
-    return hipGetLastError();
+    return launch_timed(dequant_scatter_kernel, grid, dim3(256), stream, ev.start, ev.stop, bb, kx, vx, tk, tv);
 }
 
 hipError_t launch_gather_quant(hipStream_t stream, const CodecBatch& b, const LaunchEvents& ev)
@@ -515,22 +511,12 @@ hipError_t launch_gather_quant(hipStream_t stream, const CodecBatch& b, const La
     const uint32_t hd = b.heads * b.dim;
     const uint32_t nv = b.nrec - b.n_k;
     const uint32_t kx = (2u * hd + 255u) / 256u, vx = (4u * hd + 255u) / 256u;
-    if (b.n_k + nv) {
-        const dim3 grid(kx * b.n_k + vx * nv);
-        CodecBatch bb = b;
-        bb.clock = ev.clock ? ev.clock->take(uint64_t(grid.x) * 4u) : nullptr;
-        if (ev.start || ev.stop) {
-            if (bb.bits == 8)
-                hipExtLaunchKernelGGL(quant_kernel<8>, grid, dim3(256), 0, stream, ev.start, ev.stop, 0, bb, kx, vx);
-            else
-                hipExtLaunchKernelGGL(quant_kernel<4>, grid, dim3(256), 0, stream, ev.start, ev.stop, 0, bb, kx, vx);
-        } else if (bb.bits == 8) {
-            hipLaunchKernelGGL(quant_kernel<8>, grid, dim3(256), 0, stream, bb, kx, vx);
-        } else {
-            hipLaunchKernelGGL(quant_kernel<4>, grid, dim3(256), 0, stream, bb, kx, vx);
-        }
-    }
-    return hipGetLastError();
+    if (b.n_k + nv == 0) return hipSuccess;
+    const dim3 grid(kx * b.n_k + vx * nv);
+    CodecBatch bb = b;
+    bb.clock = ev.clock ? ev.clock->take(uint64_t(grid.x) * 4u) : nullptr;
+    return launch_timed(bb.bits == 8 ? quant_kernel<8> : quant_kernel<4>, grid, dim3(256), stream, ev.start, ev.stop, bb,
+                        kx, vx);
 }
 
 }  // namespace si

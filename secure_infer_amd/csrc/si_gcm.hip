@@ -1115,9 +1115,9 @@ uint8_t* noalloc_scratch(hipStream_t stream)
     if (hipStreamIsCapturing(stream, &cs) != hipSuccess) return nullptr;
     if (cs == hipStreamCaptureStatusNone) {
         const uint64_t words = (SI_NOALLOC_CTRL_BYTES + SI_NOALLOC_ACC_BYTES) / 16u;
-        hipLaunchKernelGGL(zero_words_kernel, dim3(uint32_t((words + 255) / 256)), dim3(256), 0, stream,
-                           static_cast<uint4*>(ptr), words);
-        if (hipGetLastError() != hipSuccess) return nullptr;
+        if (launch(zero_words_kernel, dim3(uint32_t((words + 255) / 256)), dim3(256), stream, static_cast<uint4*>(ptr),
+                   words) != hipSuccess)
+            return nullptr;
         if (hipStreamSynchronize(stream) != hipSuccess) return nullptr;
     }
     ptrs[dev] = static_cast<uint8_t*>(ptr);
@@ -1171,34 +1171,27 @@ __global__ void noalloc_test_hold_kernel(uint32_t* ctrl, int hold)
 
 hipError_t launch_noalloc_acquire(hipStream_t stream, uint32_t* ctrl, uint32_t* cell)
 {
-    hipLaunchKernelGGL(noalloc_acquire_kernel, dim3(1), dim3(1), 0, stream, ctrl, cell);
-    return hipGetLastError();
+    return launch(noalloc_acquire_kernel, dim3(1), dim3(1), stream, ctrl, cell);
 }
 
 hipError_t launch_noalloc_finish(hipStream_t stream, const NoallocFinish& f)
 {
     if (f.nrec == 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(noalloc_finish_kernel, dim3(f.nrec), dim3(256), 0, stream, f);
-    return hipGetLastError();
+    return launch(noalloc_finish_kernel, dim3(f.nrec), dim3(256), stream, f);
 }
 
 hipError_t launch_noalloc_test_hold(hipStream_t stream, uint32_t* ctrl, int hold)
 {
-    hipLaunchKernelGGL(noalloc_test_hold_kernel, dim3(1), dim3(1), 0, stream, ctrl, hold);
-    return hipGetLastError();
+    return launch(noalloc_test_hold_kernel, dim3(1), dim3(1), stream, ctrl, hold);
 }
 
 // ---------------------------------------------------------------- launches
 
 template <int kMode, bool kAligned, bool kWT>
-static void launch_records(dim3 grid, dim3 block, hipStream_t stream, const LaunchEvents& ev, const GcmCtx* ctx,
-                           const RecBatch& b, const Sched& s, RecAcc* acc)
+static hipError_t launch_records(dim3 grid, dim3 block, hipStream_t stream, const LaunchEvents& ev,
+                                 const GcmCtx* ctx, const RecBatch& b, const Sched& s, RecAcc* acc)
 {
-    if (ev.start || ev.stop)
-        hipExtLaunchKernelGGL((gcm_records_kernel<kMode, kAligned, kWT>), grid, block, 0, stream, ev.start, ev.stop,
-                              0, ctx, b, s, acc);
-    else
-        hipLaunchKernelGGL((gcm_records_kernel<kMode, kAligned, kWT>), grid, block, 0, stream, ctx, b, s, acc);
+    return launch_timed(gcm_records_kernel<kMode, kAligned, kWT>, grid, block, stream, ev.start, ev.stop, ctx, b, s, acc);
 }
 
 template <int kMode>
@@ -1215,13 +1208,9 @@ static hipError_t launch_mode(hipStream_t stream, const GcmCtx* ctx, const RecBa
         e2.clock = nullptr;
         return launch_mode<kMode>(stream, ctx, b, sm, acc, aligned, e2);
     }
-    if (aligned && s.bytes % 16 == 0)
-        launch_records<kMode, true, true>(grid, block, stream, ev, ctx, b, s, acc);
-    else if (aligned)
-        launch_records<kMode, true, false>(grid, block, stream, ev, ctx, b, s, acc);
-    else
-        launch_records<kMode, false, false>(grid, block, stream, ev, ctx, b, s, acc);
-    return hipGetLastError();
+    if (aligned && s.bytes % 16 == 0) return launch_records<kMode, true, true>(grid, block, stream, ev, ctx, b, s, acc);
+    if (aligned) return launch_records<kMode, true, false>(grid, block, stream, ev, ctx, b, s, acc);
+    return launch_records<kMode, false, false>(grid, block, stream, ev, ctx, b, s, acc);
 }
 
 hipError_t launch_gcm(int mode, hipStream_t stream, const GcmCtx* ctx, const RecBatch& b,
@@ -1253,13 +1242,8 @@ hipError_t launch_release(hipStream_t stream, const GcmCtx* ctx, const RecBatch&
     chunk = (chunk + 255) / 256 * 256;
     const dim3 grid(uint32_t((nb + chunk - 1) / chunk), nrec), block(SI_RELEASE_THREADS);
     uint64_t* clock = ev.clock ? ev.clock->take(uint64_t(grid.x) * grid.y * (SI_RELEASE_THREADS / 64)) : nullptr;
-    if (ev.start || ev.stop)
-        hipExtLaunchKernelGGL(release_kernel, grid, block, 0, stream, ev.start, ev.stop, 0, ctx, b, bytes,
-                              uint32_t(chunk), aligned ? 1 : 0, gate, clock);
-    else
-        hipLaunchKernelGGL(release_kernel, grid, block, 0, stream, ctx, b, bytes, uint32_t(chunk), aligned ? 1 : 0,
-                           gate, clock);
-    return hipGetLastError();
+    return launch_timed(release_kernel, grid, block, stream, ev.start, ev.stop, ctx, b, bytes, uint32_t(chunk),
+                        aligned ? 1 : 0, gate, clock);
 }
 
 hipError_t launch_ctr(hipStream_t stream, const GcmCtx* ctx, const uint8_t* in, uint8_t* out,
@@ -1269,15 +1253,13 @@ hipError_t launch_ctr(hipStream_t stream, const GcmCtx* ctx, const uint8_t* in, 
     uint64_t grid = (nb + SI_T - 1) / SI_T;
     if (grid > 4096) grid = 4096;
     const bool aligned = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
-    hipLaunchKernelGGL(ctr_kernel, dim3(uint32_t(grid)), dim3(SI_T), 0, stream, ctx, in, out, bytes,
-                       make_uint4(iv[0], iv[1], iv[2], iv[3]), aligned ? 1 : 0);
-    return hipGetLastError();
+    return launch(ctr_kernel, dim3(uint32_t(grid)), dim3(SI_T), stream, ctx, in, out, bytes,
+                  make_uint4(iv[0], iv[1], iv[2], iv[3]), aligned ? 1 : 0);
 }
 
 hipError_t launch_ghash(hipStream_t stream, const GcmCtx* ctx, const GhashJob& j)
 {
-    hipLaunchKernelGGL(ghash_kernel, dim3(1), dim3(SI_T), 0, stream, ctx, j);
-    return hipGetLastError();
+    return launch(ghash_kernel, dim3(1), dim3(SI_T), stream, ctx, j);
 }
 
 hipError_t launch_key_fetch(hipStream_t stream, const uint8_t* key, const uint8_t* h, uint8_t* out, uint32_t* flag,
@@ -1291,8 +1273,7 @@ hipError_t launch_auth_gate(hipStream_t stream, uint8_t* data, const uint32_t* s
     uint64_t grid = (bytes + 255) / 256;
     if (grid > 1024) grid = 1024;
     if (grid == 0) grid = 1;
-    hipLaunchKernelGGL(auth_gate_kernel, dim3(uint32_t(grid)), dim3(256), 0, stream, data, status, bytes);
-    return hipGetLastError();
+    return launch(auth_gate_kernel, dim3(uint32_t(grid)), dim3(256), stream, data, status, bytes);
 }
 
 }  // namespace si

@@ -760,6 +760,12 @@ hipError_t hipLaunchKernel(const void* kernel, dim3, dim3, void** args, size_t, 
     return hipSuccess;
 }
 
+// No launch of the host code's is timed.
+hipError_t hipExtLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t, hipEvent_t, hipEvent_t, int)
+{
+    return failed(hipErrorInvalidValue);
+}
+
 // A test's own task on a stream.
 void hostsim_push(hipStream_t s, std::function<void()> f) { S(s)->push(std::move(f)); }
 
