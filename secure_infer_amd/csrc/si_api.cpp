@@ -19,6 +19,7 @@
 #include "si_layout.h"
 #include "si_host.h"
 #include "si_kernels.h"
+#include "si_launch.h"
 
 #include <openssl/core_names.h>
 #include <openssl/crypto.h>
@@ -304,7 +305,7 @@ std::unique_ptr<DevCtx> build_ctx(const uint8_t key[16], const uint8_t h[16], ui
     } im{ctx_image(key, h, npow)};
     const std::vector<uint8_t>& img = im.v;
     auto out = std::make_unique<DevCtx>();
-    if (hipMalloc(&out->dev, img.size()) != hipSuccess) return nullptr;
+    if (!si::granted(hipMalloc(&out->dev, img.size()))) return nullptr;
     if (hipMemcpy(out->dev, img.data(), img.size(), hipMemcpyHostToDevice) != hipSuccess) return nullptr;
     out->npow = npow;
     memcpy(out->key, key, 16);
@@ -523,7 +524,7 @@ si::RecAcc* workspace(Workspace& w, hipStream_t stream, size_t nrec)
     }
     size_t cap = 256;
     while (cap < nrec) cap *= 2;
-    if (hipMalloc(&w.acc, cap * sizeof(si::RecAcc)) != hipSuccess) return nullptr;
+    if (!si::granted(hipMalloc(&w.acc, cap * sizeof(si::RecAcc)))) return nullptr;
     if (hipMemset(w.acc, 0, cap * sizeof(si::RecAcc)) != hipSuccess) return nullptr;
     w.cap = cap;
     return w.acc;
@@ -540,7 +541,7 @@ uint4* park_area(Workspace& w, hipStream_t stream, size_t nwg)
         w.park = nullptr;
         w.park_cap = 0;
     }
-    if (hipMalloc(&w.park, need * sizeof(uint4)) != hipSuccess) return nullptr;
+    if (!si::granted(hipMalloc(&w.park, need * sizeof(uint4)))) return nullptr;
     w.park_cap = need;
     return w.park;
 }
@@ -801,8 +802,8 @@ std::unique_ptr<DevCtx> build_ctx_on_device(hipStream_t stream, const uint8_t* d
     uint32_t* d_te0 = nullptr;
     auto out = std::make_unique<DevCtx>();
     const size_t bytes = sizeof(si::GcmCtx) + size_t(npow) * 16;
-    bool ok = hipMalloc(reinterpret_cast<void**>(&out->dev), bytes) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void**>(&d_te0), sizeof(te0)) == hipSuccess &&
+    bool ok = si::granted(hipMalloc(reinterpret_cast<void**>(&out->dev), bytes)) &&
+              si::granted(hipMalloc(reinterpret_cast<void**>(&d_te0), sizeof(te0))) &&
               hipMemcpyAsync(d_te0, te0, sizeof(te0), hipMemcpyHostToDevice, stream) == hipSuccess &&
               si::launch_ctx_build(stream, dev_key, d_te0, out->dev, npow) == hipSuccess &&
               hipStreamSynchronize(stream) == hipSuccess;
@@ -862,10 +863,10 @@ int secure_infer_gpu_session_agree(uint64_t session_nonce, uint64_t max_record_b
         // A private stream, as the reference's setup stream: nothing the
         // caller has queued is waited for.
         if (hipStreamCreateWithFlags(&b.stream, hipStreamNonBlocking) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void**>(&b.io), sizeof(si::AgreeIo)) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void**>(&b.key), 16) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void**>(&b.pool), SI_AGREE_POOL_WORDS * 4) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void**>(&b.counter), 4) != hipSuccess ||
+            !si::granted(hipMalloc(reinterpret_cast<void**>(&b.io), sizeof(si::AgreeIo))) ||
+            !si::granted(hipMalloc(reinterpret_cast<void**>(&b.key), 16)) ||
+            !si::granted(hipMalloc(reinterpret_cast<void**>(&b.pool), SI_AGREE_POOL_WORDS * 4)) ||
+            !si::granted(hipMalloc(reinterpret_cast<void**>(&b.counter), 4)) ||
             hipMemcpyAsync(b.io, &io, sizeof(io), hipMemcpyHostToDevice, b.stream) != hipSuccess ||
             si::launch_agree(b.stream, field(b.io, offsetof(si::AgreeIo, host_public)),
                              field(b.io, offsetof(si::AgreeIo, challenge)), seed, b.pool, b.counter, b.key,
@@ -940,7 +941,7 @@ int64_t secure_infer_test_context_image(const uint8_t key[16], uint64_t max_reco
     hipStream_t st = nullptr;
     uint8_t* d_key = nullptr;
     bool ok = hipStreamCreateWithFlags(&st, hipStreamNonBlocking) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void**>(&d_key), 16) == hipSuccess &&
+              si::granted(hipMalloc(reinterpret_cast<void**>(&d_key), 16)) &&
               hipMemcpyAsync(d_key, key, 16, hipMemcpyHostToDevice, st) == hipSuccess;
     std::unique_ptr<DevCtx> c = ok ? build_ctx_on_device(st, d_key, npow) : nullptr;
     ok = c && hipMemcpy(out, c->dev, bytes, hipMemcpyDeviceToHost) == hipSuccess;
@@ -953,7 +954,7 @@ int secure_infer_test_x25519(const uint8_t scalar[32], const uint8_t u[32], uint
 {
     if (!scalar || !u || !out) return -1;
     uint8_t* d = nullptr;
-    bool ok = hipMalloc(reinterpret_cast<void**>(&d), 96) == hipSuccess &&
+    bool ok = si::granted(hipMalloc(reinterpret_cast<void**>(&d), 96)) &&
               hipMemcpy(d, scalar, 32, hipMemcpyHostToDevice) == hipSuccess &&
               hipMemcpy(d + 32, u, 32, hipMemcpyHostToDevice) == hipSuccess &&
               si::launch_x25519_test(nullptr, d, d + 32, d + 64) == hipSuccess &&
@@ -968,7 +969,7 @@ int secure_infer_test_blake2b(const uint8_t* key, uint32_t key_len, const uint8_
     if ((key_len && !key) || key_len > 64 || (msg_len && !msg) || !out || out_len == 0 || out_len > 64) return -1;
     uint8_t* d = nullptr;
     const uint64_t n = 64 + 64 + msg_len + 1;
-    bool ok = hipMalloc(reinterpret_cast<void**>(&d), n) == hipSuccess &&
+    bool ok = si::granted(hipMalloc(reinterpret_cast<void**>(&d), n)) &&
               (key_len == 0 || hipMemcpy(d, key, key_len, hipMemcpyHostToDevice) == hipSuccess) &&
               (msg_len == 0 || hipMemcpy(d + 128, msg, msg_len, hipMemcpyHostToDevice) == hipSuccess) &&
               si::launch_blake2b_test(nullptr, d, key_len, d + 128, msg_len, d + 64, out_len) == hipSuccess &&
@@ -1572,7 +1573,7 @@ int secure_infer_gpu_key_agreement_do(hipStream_t stream, void* host_public, voi
     // allocated, filled, hashed, zeroed and freed in stream order.
     const size_t pool_bytes = size_t(SI_AGREE_POOL_WORDS) * 4 + 16;
     uint32_t* pool = nullptr;
-    if (hipMallocAsync(reinterpret_cast<void**>(&pool), pool_bytes, stream) != hipSuccess) {
+    if (!si::granted(hipMallocAsync(reinterpret_cast<void**>(&pool), pool_bytes, stream))) {
         OPENSSL_cleanse(seed.b, sizeof(seed.b));
         return -1;
     }

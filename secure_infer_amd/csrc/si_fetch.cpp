@@ -6,6 +6,7 @@
 #include <new>
 
 #include "si_kernels.h"
+#include "si_launch.h"
 
 namespace si {
 
@@ -66,10 +67,7 @@ Slot* take_slot()
     }
     if (free_slot && !free_slot->box) {
         void* b = nullptr;
-        if (hipHostMalloc(&b, sizeof(Box), hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
+        if (!granted(hipHostMalloc(&b, sizeof(Box), hipHostMallocPortable | hipHostMallocMapped))) return nullptr;
         free_slot->box = new (b) Box();
     }
     return free_slot;

@@ -43,6 +43,7 @@
 //  * Every block id is range-checked on the host before any work: a swap
 //    with a host block or device slot outside its pool is refused (-1).
 #include "si_host.h"
+#include "si_launch.h"
 
 #include <openssl/evp.h>
 #include <sched.h>
@@ -359,8 +360,8 @@ struct Mirror {
             host = nullptr;
             dev = nullptr;
             cap = 0;
-            if (hipHostMalloc(reinterpret_cast<void**>(&host), need, hipHostMallocDefault) != hipSuccess ||
-                hipMalloc(reinterpret_cast<void**>(&dev), need) != hipSuccess)
+            if (!si::granted(hipHostMalloc(reinterpret_cast<void**>(&host), need, hipHostMallocDefault)) ||
+                !si::granted(hipMalloc(reinterpret_cast<void**>(&dev), need)))
                 return false;
             cap = need;
         }
@@ -368,7 +369,7 @@ struct Mirror {
             if (stage) (void)hipFree(stage);
             stage = nullptr;
             stage_cap = 0;
-            if (hipMalloc(reinterpret_cast<void**>(&stage), stage_need) != hipSuccess) return false;
+            if (!si::granted(hipMalloc(reinterpret_cast<void**>(&stage), stage_need))) return false;
             stage_cap = stage_need;
         }
         return true;
@@ -484,7 +485,7 @@ std::unique_ptr<StatusBuf> take_status(DeviceState* ds, size_t words)
     }
     auto b = std::make_unique<StatusBuf>();
     const size_t cap = std::max<size_t>(1024, (words + 1023) / 1024 * 1024);
-    if (hipHostMalloc(reinterpret_cast<void**>(&b->host), cap * 4, hipHostMallocDefault) != hipSuccess ||
+    if (!si::granted(hipHostMalloc(reinterpret_cast<void**>(&b->host), cap * 4, hipHostMallocDefault)) ||
         hipHostGetDevicePointer(reinterpret_cast<void**>(&b->dev), b->host, 0) != hipSuccess ||
         hipEventCreateWithFlags(&b->ready, hipEventDisableTiming) != hipSuccess)
         return nullptr;
@@ -718,7 +719,7 @@ uint8_t* take_pf_buffer(size_t need, size_t& cap)
     for (uint8_t* p : drop) (void)hipHostFree(p);
     if (!fits) return nullptr;
     uint8_t* p = nullptr;
-    if (hipHostMalloc(reinterpret_cast<void**>(&p), need, hipHostMallocDefault) != hipSuccess) {
+    if (!si::granted(hipHostMalloc(reinterpret_cast<void**>(&p), need, hipHostMallocDefault))) {
         std::lock_guard<std::mutex> g(g_pf_lock);
         g_pf_bytes -= need;
         return nullptr;

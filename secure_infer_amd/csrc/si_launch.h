@@ -1,4 +1,4 @@
-// Kernel launches that report their own status.
+// Kernel launches and allocations that report their own status.
 #pragma once
 
 #include <hip/hip_ext.h>
@@ -38,6 +38,14 @@ template <class... P, class... A>
 hipError_t launch(void (*kernel)(P...), dim3 grid, dim3 block, hipStream_t stream, A&&... a)
 {
     return launch_timed(kernel, grid, block, stream, nullptr, nullptr, std::forward<A>(a)...);
+}
+
+// An allocation's status, for a caller that reports a refusal itself: none stays
+// behind as the thread's last error.
+inline bool granted(hipError_t e)
+{
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
 }
 
 }  // namespace si

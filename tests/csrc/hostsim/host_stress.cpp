@@ -43,7 +43,7 @@
 #include "si_oracle.h"
 
 extern "C" size_t hostsim_reload_log(uint32_t layer, uint64_t* out, size_t cap);
-extern "C" void hostsim_refuse(const char* call);
+extern "C" void hostsim_refuse(const char* call, int skip = 0);
 void hostsim_push(hipStream_t s, std::function<void()> f);
 void hostsim_fetch_hook(std::function<void(const uint8_t*)> f);
 size_t hostsim_pinned_copies(const uint8_t* b, size_t n);
@@ -575,6 +575,27 @@ void fetch_not_seen_to_end()
     (void)hipStreamDestroy(sb);
 }
 
+// Refused allocations fail the call and leave no pending HIP error: a
+// session's context, a kernel-level call's context and its stream's workspace.
+void refused_allocations()
+{
+    si_session* sess = nullptr;
+    hostsim_refuse("hipMalloc");
+    CHECK(secure_infer_gpu_session_create(kKey, kSalt, 1, 4096, &sess) == -1, "session_create");
+    CHECK(hipGetLastError() == hipSuccess, "session_create: an error stays pending");
+    const KeyPair k(5);
+    uint8_t* d = nullptr;
+    CHECK(hipMalloc(&d, 64) == hipSuccess, "hipMalloc");
+    for (int skip = 0; skip < 2; ++skip) {  // the context, then the workspace
+        hostsim_refuse("hipMalloc", skip);
+        CHECK(secure_infer_gpu_gcm_encrypt_tag_do(nullptr, d, k.dev, k.dev + 16, d + 16, d + 32, 16, 1, 2, 3, 2, nullptr,
+                                                  0) == -1, "refused allocation %d", skip);
+        CHECK(hipGetLastError() == hipSuccess, "refused allocation %d: an error stays pending", skip);
+    }
+    hostsim_refuse("");
+    (void)hipFree(d);
+}
+
 int main(int argc, char** argv)
 {
     if (argc > 2 && std::string(argv[1]) == "key_fetch") {
@@ -582,6 +603,7 @@ int main(int argc, char** argv)
         if (what == "pending_error") fetch_with_a_pending_error();
         else if (what == "unseen_end") fetch_not_seen_to_end();
         else if (what == "declined") declined_fetches();
+        else if (what == "refused_allocations") refused_allocations();
         else return 2;
         hipDeviceSynchronize();
         if (g_failures.load()) return 1;

@@ -197,19 +197,25 @@ hipError_t failed(hipError_t e)
     return e;
 }
 
-// The calling thread's next call of this name fails (hostsim_refuse).
+// The calling thread's next call of this name, after `t_skip` more, fails
+// (hostsim_refuse).
 thread_local std::string t_refused;
+thread_local int t_skip = 0;
 
 bool refused(const char* call)
 {
-    if (t_refused != call) return false;
+    if (t_refused != call || t_skip-- > 0) return false;
     t_refused.clear();
     return true;
 }
 
 }  // namespace
 
-extern "C" void hostsim_refuse(const char* call) { t_refused = call; }
+extern "C" void hostsim_refuse(const char* call, int skip)
+{
+    t_refused = call;
+    t_skip = skip;
+}
 
 hipError_t hipGetDevice(int* dev)
 {
