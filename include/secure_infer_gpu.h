@@ -492,6 +492,9 @@ int secure_infer_test_noalloc_hold(hipStream_t stream, int hold);
  * verification alone, so a test can see that it writes nothing but
  * statuses); 0 disarms.  0 or -1.  Production code never calls it. */
 int secure_infer_test_strict_phases(int n);
+/* Test-only (no reference counterpart): how many kernel-level calls so far got
+ * their key from the fetch kernel (the others copied it). */
+uint64_t secure_infer_test_key_fetches(void);
 int secure_infer_test_x25519(const uint8_t scalar[32], const uint8_t u[32], uint8_t out[32]);
 int secure_infer_test_blake2b(const uint8_t* key, uint32_t key_len, const uint8_t* msg, uint64_t msg_len,
                               uint8_t* out, uint32_t out_len);

@@ -87,6 +87,7 @@ SIGNATURES = {
     "secure_infer_test_tamper_agree": ([_u32], _i),
     "secure_infer_test_noalloc_hold": ([_v, _i], _i),
     "secure_infer_test_strict_phases": ([_i], _i),
+    "secure_infer_test_key_fetches": ([], _u64),
     "secure_infer_retire_transfer_prefetches": ([], None),
     "secure_infer_invalidate_transfer_prefetches": ([], None),
     "secure_infer_get_transfer_prefetch_stats": ([ct.POINTER(_u64)] * 3, None),

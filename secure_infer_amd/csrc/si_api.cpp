@@ -1289,6 +1289,8 @@ int secure_infer_gpu_clock_rate_khz(uint64_t* khz)
     return 0;
 }
 
+uint64_t secure_infer_test_key_fetches(void) { return si::key_fetches(); }
+
 int secure_infer_test_strict_phases(int n)
 {
     if (n < 0) return -1;

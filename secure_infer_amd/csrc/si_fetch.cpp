@@ -1,6 +1,7 @@
 // The host's read of a device-resident key and H (the kernel-level calls).
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <mutex>
 #include <new>
@@ -44,6 +45,7 @@ constexpr int kSlots = 16;
 std::mutex g_boxes_lock;
 Slot g_boxes[kSlots];
 uint32_t g_seq = 0;  // never 0 in a fetch
+std::atomic<uint64_t> g_fetches{0};
 
 bool landed(const Box* b, uint32_t seq) { return __atomic_load_n(&b->flag, __ATOMIC_ACQUIRE) == seq; }
 
@@ -124,7 +126,10 @@ hipError_t fetch_key(hipStream_t stream, const void* key, const void* h, uint8_t
     if (e == hipSuccess)
         for (int k = 0; k < (h ? 32 : 16); ++k) out[k] = w[k];
     wipe(box);
+    if (e == hipSuccess) g_fetches.fetch_add(1, std::memory_order_relaxed);
     return e;
 }
+
+uint64_t key_fetches() { return g_fetches.load(std::memory_order_relaxed); }
 
 }  // namespace si

@@ -172,6 +172,8 @@ hipError_t launch_ctr(hipStream_t stream, const GcmCtx* ctx, const uint8_t* in, 
 // that are not the current device's own memory, for a stream under capture and
 // where there is no pinned memory to fetch into.
 hipError_t fetch_key(hipStream_t stream, const void* key, const void* h, uint8_t out[32]);
+// Fetches that returned a key so far (tests).
+uint64_t key_fetches();
 // One wave: key[0..16) and, unless null, h[0..16) to out[0..16) and out[16..32),
 // then seq to *flag (out and flag: device addresses of pinned host memory).
 hipError_t launch_key_fetch(hipStream_t stream, const uint8_t* key, const uint8_t* h, uint8_t* out, uint32_t* flag,

@@ -575,6 +575,40 @@ void fetch_not_seen_to_end()
     (void)hipStreamDestroy(sb);
 }
 
+// Threads with their own streams and keys, one of them on a stream that is held
+// over each second fetch (so that the host waits for the stream, and in each
+// fourth the wait fails): each gets its own key, and none stays behind.
+void fetches_from_threads()
+{
+    std::vector<std::unique_ptr<KeyPair>> keys;
+    for (uint32_t i = 0; i < 4; ++i) keys.push_back(std::make_unique<KeyPair>(10 + i));
+    std::atomic<int> failed{0};
+    std::vector<std::thread> ts;
+    for (int i = 0; i < 4; ++i)
+        ts.emplace_back([&, i] {
+            hipStream_t s = nullptr;
+            CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess, "stream");
+            for (int n = 0; n < 60; ++n) {
+                if (i == 0 && n % 2) hostsim_push(s, [] { std::this_thread::sleep_for(std::chrono::milliseconds(5)); });
+                if (i == 0 && n % 4 == 3) hostsim_refuse("hipStreamSynchronize");
+                uint8_t out[32];
+                const hipError_t e = keys[i]->fetch(s, out);
+                hostsim_refuse("");
+                if (e == hipSuccess) CHECK(!memcmp(out, keys[i]->bytes, 32), "thread %d, fetch %d: another key", i, n);
+                else failed.fetch_add(1);
+                CHECK(e == hipSuccess || (i == 0 && n % 4 == 3), "thread %d, fetch %d failed", i, n);
+            }
+            CHECK(hipStreamSynchronize(s) == hipSuccess, "sync");
+            (void)hipStreamDestroy(s);
+        });
+    for (auto& t : ts) t.join();
+    CHECK(keys[1]->fetched(nullptr), "a last fetch");
+    CHECK(hipDeviceSynchronize() == hipSuccess, "sync");
+    for (auto& k : keys) CHECK(hostsim_pinned_copies(k->bytes, 16) == 0, "a key stays in pinned memory");
+    CHECK(failed.load() > 0 && si::key_fetches() == uint64_t(241 - failed.load()), "%d failed, %llu fetched",
+          failed.load(), static_cast<unsigned long long>(si::key_fetches()));
+}
+
 // Refused allocations fail the call and leave no pending HIP error: a
 // session's context, a kernel-level call's context and its stream's workspace.
 void refused_allocations()
@@ -603,6 +637,7 @@ int main(int argc, char** argv)
         if (what == "pending_error") fetch_with_a_pending_error();
         else if (what == "unseen_end") fetch_not_seen_to_end();
         else if (what == "declined") declined_fetches();
+        else if (what == "threads") fetches_from_threads();
         else if (what == "refused_allocations") refused_allocations();
         else return 2;
         hipDeviceSynchronize();

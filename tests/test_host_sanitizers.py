@@ -83,14 +83,15 @@ def test_d2h_authentication_failure_handling(abort):
         assert r.returncode == 0 and "D2H_FAILURE_REPORTED" in r.stdout, report[-4000:]
 
 
-@pytest.mark.parametrize("what", ["pending_error", "unseen_end", "declined", "refused_allocations"])
+@pytest.mark.parametrize("what", ["pending_error", "unseen_end", "declined", "threads", "refused_allocations"])
 @pytest.mark.parametrize("san", ["thread", "address"])
 def test_key_fetch(san, what):
     """The host's read of a device-resident key (si_fetch.cpp): an earlier
     call's pending error does not abandon a queued fetch; a fetch whose end was
     not seen keeps its box to itself until it ends; a declined fetch leaves no
     pending error behind, and neither does a call that fails because an
-    allocation was refused."""
+    allocation was refused; threads with their own streams and keys, one of whose
+    waits fail now and then, each get their own key."""
     r = subprocess.run([str(build(san)), "key_fetch", what], capture_output=True, text=True, timeout=120,
                        env={**os.environ, "TSAN_OPTIONS": "halt_on_error=1", "ASAN_OPTIONS": "halt_on_error=1"})
     assert r.returncode == 0 and "KEY_FETCH_OK" in r.stdout, (r.stdout + r.stderr)[-4000:]
