@@ -649,9 +649,11 @@ __device__ __forceinline__ void gcm_records_body(const GcmCtx* __restrict__ ctx,
 
     // This workgroup's share of the records' concatenated rows: rows
     // [qa0, qb0) of record r0 and, with two segments, [0, qb1) of r0 + 1.  The
-    // laid-out starts are 32-bit, so their record takes a 32-bit division (the
-    // emulated 64-bit one sat on the set-up's critical path); the 64-bit form
-    // is for batches of more than SI_MAX_WG shares only.
+    // laid-out starts are 32-bit, so their record takes a 32-bit division
+    // instead of the emulated 64-bit one (MI355X, this alone: 96 records of 256
+    // KiB 30.8 -> 30.6 us, 512 of 32 KiB 28.2 -> 28.1, two and 32 records of
+    // 256 KiB 0.1 us slower); the 64-bit form is for batches of more than
+    // SI_MAX_WG shares only.
     uint32_t r0, qa0, len;
     if (sch.use_starts) {
         const uint32_t g0 = sch.starts[blockIdx.x];
@@ -810,10 +812,10 @@ __device__ __forceinline__ void gcm_records_body(const GcmCtx* __restrict__ ctx,
         // the record's accumulator per share instead of five.  The atomics of
         // a record's shares queue up on its one line, which bounds a launch
         // of few records (two 256-KiB records in 44 shares: 2.9 us from the
-        // last barrier to the flags below, of 13.9 us).  MI355X, with the
-        // 32-bit share starts above, four 32-bit XORs -> these: that launch
-        // 13.9 -> 12.6 us, 32 records of 256 KiB 18.4 -> 18.1, 512 of 32 KiB
-        // 28.1 -> 27.7, 96 of 256 KiB 30.3 -> 30.2.
+        // last barrier to the flags below, of 13.9 us).  MI355X, four 32-bit
+        // XORs -> these, the 32-bit share starts above on both sides: that
+        // launch 14.0 -> 12.7 us, 32 records of 256 KiB 18.7 -> 18.4, 512 of 32
+        // KiB 28.1 -> 27.9, 96 of 256 KiB 30.6 both.
         const uint32_t s = tid >> 1, h = tid & 1u;
         const uint32_t qa = s ? 0u : qa0, qb = s ? qb1 : qb0;
         const auto half = [&](const uint4* q) { return reinterpret_cast<const uint64_t*>(q)[h]; };
